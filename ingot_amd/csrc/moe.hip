@@ -12,7 +12,7 @@
 //     returns when the slot is unused, so the host never waits for the routing. A slot's tokens are gathered through
 //     a row map: the round's rows for gate|up, the expert's own pair rows for down.
 //   - Weights stream as 16-row × 128-K tiles, one 1024-byte dwordx4 load per wave and tile (the dense qmm's layout);
-//     a workgroup of one wave takes four tiles over all of K (few K-blocks), or four waves split K over two tiles,
+//     a workgroup of one wave takes four tiles over all of K (few K-blocks), or four waves split K over one to four,
 //     added in wave order in LDS (many K-blocks).
 //   - int4 g64: bf16 MFMA on 128 + q with the affine map applied per group (as the dense qmm). MXFP4: a pair of e2m1
 //     codes becomes its exact fp16 values with one v_cvt_scalef32_pk_f16_fp4; the MFMA runs in fp16 against fp16
@@ -590,50 +590,53 @@ int launch_gather(ih_ctx* c, const ih_qmat* W, const GatherParams& base, int slo
   IH_CHECK(size_t(W->E) * p.tiles_per_e * 1024u < (size_t(1) << 31), IH_EINVAL,
            "gathered qmm: stacked matrix above 2 GiB");
   TimedLaunch tl(c, TC_MOE, bytes);
-  // Waves per workgroup (K split), row tiles per workgroup and ring depth, measured on the MoE configurations (i.i.d.
-  // routing, MoE kernels per step). Many slots: with K at most 16 K-blocks (E128 top-8, K = 2048 and 768) one wave
-  // per workgroup over four tiles (3.27 ms) beats two waves over four tiles (3.30), over two tiles (3.72) and four
-  // waves over two (3.95) or one (5.13); with more K-blocks four waves split K over two tiles or more. A slot holds few pairs, so a workgroup's life is a
-  // few memory latencies and the rate is set by how much each wave streams behind them: longer waves win until the
-  // registers cost waves per SIMD (eight tiles: 171 VGPRs, 3.53 ms; a ring of two or three stages: 4.47, 5.70). A
-  // single slot (a router, or one expert) has few workgroups; there K is split over waves and every K-block of a
-  // wave is requested at entry.
+  // Waves per workgroup (K split), row tiles per workgroup and ring depth. The waves order a row's sum, so they follow the
+  // matrix only, never the number of routed slots (a token must give the same bits decoded alone and in a block): with K
+  // at most 16 K-blocks one wave, else four. Measured on the MoE configurations (i.i.d. routing, MoE kernels per step),
+  // many slots: with K at most 16 K-blocks (E128 top-8, K = 2048 and 768) one wave per workgroup over four tiles (3.27 ms)
+  // beats two waves over four tiles (3.30), over two tiles (3.72) and four waves over two (3.95) or one (5.13). With more
+  // K-blocks four waves over two tiles beat two waves (MXFP4, K = 2880, 32 experts top-4: 5760 rows, 5 and 9 rows a block,
+  // 27.2 and 36.0 against 29.0 and 38.2 µs; 2880 rows 17.5 and 20.4 against 18.2 and 20.0, one row 9.3 against 12.1, 17
+  // rows 24.4 against 27.8). A slot holds few pairs, so a workgroup's life is a few memory latencies and the rate is set by
+  // how much each wave streams behind them: longer waves win until the registers cost waves per SIMD (eight tiles: 171
+  // VGPRs, 3.53 ms; a ring of two or three stages: 4.47, 5.70). A single slot (a router, or one expert) has few
+  // workgroups; every K-block of a wave, up to four, is requested at entry there, and K is split in two where the launch
+  // is always a single slot (one row of top-1 experts, 1536 × 2048: 9.0 µs in one wave, 8.1 in two).
   // Only tiles with a live row are launched (rows are padded to 256 in memory, so the tiles of a group past N stay
   // inside the matrix: their rows read as the zero padding and are not stored).
   const int tiles = (W->N + 15) / 16;
-  int GKW, R = 1, D = 1;
+  const bool routed = p.slots || p.entries;  // as many slots as the block's rows choose experts
+  const int GKW = W->nkb > 16 ? 4 : routed ? 1 : 2;
+  const int kpw = (W->nkb + GKW - 1) / GKW;
+  int R = 1, D = 1;
   if (slots == 1) {
-    GKW = W->nkb <= 16 ? 2 : 4;
-    const int kpw = (W->nkb + GKW - 1) / GKW;
     D = kpw <= 1 ? 1 : (kpw <= 2 ? 2 : 4);
   } else if (W->nkb <= 16) {
-    GKW = 1;
     R = 4;
   } else {
-    GKW = 4;
     if (((tiles + 1) / 2) * slots >= 2 * c->cu_count) R = 2;
-    if (W->format == QF_MXFP4 && R == 2) {
-      // With the one-instruction decode: 32 slots of 360 tiles (gate|up, K = 2880) 47.8 µs at (R, waves) = (2, 4), 45.8
-      // at (4, 4), 46.4 at (4, 2); of 180 tiles (down) 23.7 at (2, 4), 21.8 at (2, 2), 23.6 at (4, 4).
-      if (((tiles + 3) / 4) * slots >= 8 * c->cu_count) R = 4;
-      else GKW = 2;
-    }
+    // Four tiles where that still leaves eight workgroups a CU (the one-instruction decode leaves the registers for it;
+    // 8192 × 4096, 9 and 17 rows: 59.2 and 86.9 µs against 63.1 and 91.4).
+    if (W->format == QF_MXFP4 && ((tiles + 3) / 4) * slots >= 8 * c->cu_count) R = 4;
   }
-  const int kpw = (W->nkb + GKW - 1) / GKW;
   p.trips = (kpw + D - 1) / D;
   const dim3 grid((tiles + R - 1) / R, slots);
+  bool ok = false;
+#define IH_GATHER_FMT(FMT_, R_, D_, W_)                                                                             \
+  tlaunch(tl, qmm_gather_kernel<FMT_, R_, D_, W_>, grid, dim3(64 * W_), 0, c->stream, p), ok = true
 #define IH_GATHER_LAUNCH(R_, D_, W_)                                                                                \
-  if (R == R_ && D == D_ && GKW == W_) {                                                                          \
-    if (W->format == QF_MXFP4)                                                                                    \
-      tlaunch(tl, qmm_gather_kernel<QF_MXFP4, R_, D_, W_>, grid, dim3(64 * W_), 0, c->stream, p);                 \
-    else if (x_f16)                                                                                               \
-      tlaunch(tl, qmm_gather_kernel<GF_INT4_F16, R_, D_, W_>, grid, dim3(64 * W_), 0, c->stream, p);              \
-    else                                                                                                          \
-      tlaunch(tl, qmm_gather_kernel<QF_INT4, R_, D_, W_>, grid, dim3(64 * W_), 0, c->stream, p);                  \
+  if (R == R_ && D == D_ && GKW == W_) {                                                                            \
+    if (W->format == QF_MXFP4) IH_GATHER_FMT(QF_MXFP4, R_, D_, W_);                                                 \
+    else if (x_f16) IH_GATHER_FMT(GF_INT4_F16, R_, D_, W_);                                                         \
+    else IH_GATHER_FMT(QF_INT4, R_, D_, W_);                                                                        \
   }
-  IH_GATHER_LAUNCH(1, 1, 2) IH_GATHER_LAUNCH(1, 2, 2) IH_GATHER_LAUNCH(1, 4, 2) IH_GATHER_LAUNCH(1, 1, 4)
-  IH_GATHER_LAUNCH(1, 2, 4) IH_GATHER_LAUNCH(1, 4, 4) IH_GATHER_LAUNCH(2, 1, 4) IH_GATHER_LAUNCH(4, 1, 1) IH_GATHER_LAUNCH(2, 1, 2) IH_GATHER_LAUNCH(4, 1, 4)
+  IH_GATHER_LAUNCH(1, 1, 1) IH_GATHER_LAUNCH(1, 2, 1) IH_GATHER_LAUNCH(1, 4, 1) IH_GATHER_LAUNCH(4, 1, 1)
+  IH_GATHER_LAUNCH(1, 1, 2) IH_GATHER_LAUNCH(1, 2, 2) IH_GATHER_LAUNCH(1, 4, 2)
+  IH_GATHER_LAUNCH(1, 1, 4) IH_GATHER_LAUNCH(1, 4, 4) IH_GATHER_LAUNCH(2, 1, 4)
+  if (W->format == QF_MXFP4 && R == 4 && GKW == 4) IH_GATHER_FMT(QF_MXFP4, 4, 1, 4);
 #undef IH_GATHER_LAUNCH
+#undef IH_GATHER_FMT
+  IH_CHECK(ok, IH_EINVAL, "gathered qmm: launch shape not instantiated");
   IH_HIP(hipGetLastError());
   return IH_OK;
 }

@@ -367,3 +367,23 @@ def test_rows_do_not_depend_on_the_attention_kernel(ctx, shape, chunk):
     finally:
         kv.free()
         m.free()
+
+
+# MXFP4 experts over 23 K-blocks: the sum over K is split between the waves of a workgroup.
+MOEX23 = dict(MOEX, n_layers=2, hidden=2880, n_experts=32, expert_intermediate=2880, iid_routing=1)
+
+
+@pytest.mark.parametrize("shape", [MOEX23], ids=["moe-mxfp4-k2880"])
+def test_rows_do_not_depend_on_the_launch_shapes(ctx, shape):
+    """A row's logits have the same bits in a full block and in every shorter one."""
+    d, m, kv = make(ctx, shape)
+    try:
+        toks = np.random.default_rng(3).integers(0, d.vocab, size=17).astype(np.uint32)
+        _, full = kv.verify(toks, want_logits=True)
+        assert np.all(np.isfinite(full))
+        for B in (16, 1, 2, 5, 6, 9):
+            _, part = kv.verify(toks[:B], want_logits=True)
+            assert np.array_equal(part.view(np.uint32), full[:B].view(np.uint32)), B
+    finally:
+        kv.free()
+        m.free()

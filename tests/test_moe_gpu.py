@@ -236,3 +236,39 @@ def test_mxfp4_special_scales_and_row_alignment(ctx, N, K, off, pad):
     assert np.array_equal(np.isnan(got), np.isnan(ref))
     ok = ~np.isnan(ref)
     assert np.abs(got[ok] - ref[ok]).max() <= 2e-5 * np.abs(ref[ok]).max()
+
+
+# (format, E, top k, N, K): gate|up and down of the two MoE configurations, few tiles over many K-blocks, and top-1
+# experts, where one row is a single slot.
+BLOCKS = [("mxfp4", 32, 4, 5760, 2880), ("mxfp4", 32, 4, 2880, 2880), ("mxfp4", 16, 2, 272, 2880),
+          ("mxfp4", 16, 1, 2880, 2880), ("int4", 128, 8, 1536, 2048), ("int4", 32, 4, 1408, 2880),
+          ("int4", 8, 1, 256, 1024)]
+
+
+@pytest.mark.parametrize("fmt,E,K,N,D", BLOCKS, ids=["-".join(map(str, b)) for b in BLOCKS])
+def test_expert_rows_do_not_depend_on_the_block(ctx, fmt, E, K, N, D):
+    """A row's product with each of its experts has the same bits whatever the number of rows that are routed with it
+    (one row: plain decoding; 17: a verify block): the order of its sum over K is the matrix's own."""
+    g = rng(N + D + K)
+    w = g.integers(0, 2**32, size=(E, N, D // 8), dtype=np.uint32)
+    if fmt == "int4":
+        s = oracle.f32_to_bf16(np.abs(g.normal(0, 0.02, size=(E, N, D // 64))).astype(np.float32))
+        W = QMat.int4(ctx, w, s, oracle.f32_to_bf16(-8.0 * oracle.bf16_to_f32(s)))
+    else:
+        W = QMat.mxfp4(ctx, w, g.integers(119, 126, size=(E, N, D // 32), dtype=np.uint8))
+    xb, _ = bf16_normal(g, (17, D))
+    logits = g.normal(0, 1, size=(17, E)).astype(np.float32)
+    try:
+        want = None
+        for rows in (17, 1, 2, 3, 5, 6, 7, 9, 16):
+            dl, dx = ctx.to_device(logits[:rows].copy()), ctx.to_device(xb[:rows].copy())
+            R = Routing(ctx, rows, K, E).route(dl, E)
+            y, row_pair = R.gathered(W, dx), R.download()["row_pair"]
+            for x in (R, dl, dx):
+                x.free()
+            got = y[row_pair]  # [rows, K, N]
+            if want is None:
+                want = got
+            assert np.array_equal(got.view(np.uint32), want[:rows].view(np.uint32)), rows
+    finally:
+        W.free()
