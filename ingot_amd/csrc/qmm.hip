@@ -175,7 +175,8 @@ static QmmShape qmm_shape_sym(int Npad, int nkb, int M) {
   // K-block counts without a fitting factor: one split whose last wave runs past the end by less than its kpw. One token
   // tile leaves less x to share, and two row tiles per wave win there (K = 2880, 9 rows: 32000 11.1 against 12.5 µs, 50257
   // 20.7 against 23.9, 201088 74.7 against 80.4; 17 rows: 20.0, 36.1 and 125.8 against 14.9, 32.1 and 101.5). Only the
-  // row tiles follow M: the waves and their K-blocks, which order a row's sums, stay.
+  // row tiles follow M (not for the residual epilogue, see qmm_setup): the waves and their K-blocks, which order a row's
+  // sums, stay.
   for (int R : rp)
     if (R)
       for (const auto& c : kQmmShapes) {
@@ -226,11 +227,15 @@ static int ensure_qpart(ih_ctx* c, size_t bytes) {
   return IH_OK;
 }
 
-// The launch's shape (an override of the matrix size first), its K split and the weight side of its parameters.
-static int qmm_setup(ih_ctx* c, const ih_qmat* W, int expert, int M, bool rows, QmmShape& sh, QmmParams& p, dim3& grid) {
+// The launch's shape (an override of the matrix size first), its K split and the weight side of its parameters. `rows`:
+// the caller's rows (qmm_rows.hip).
+static int qmm_setup(ih_ctx* c, const ih_qmat* W, int expert, int M, int mode, bool rows, QmmShape& sh, QmmParams& p,
+                     dim3& grid) {
   IH_CHECK(W->format == QF_INT4, IH_EINVAL, "qmm: int4 matrix expected");
   IH_CHECK(M >= 1 && M <= MAX_TOK, IH_EINVAL, "qmm: M must be in 1..32");
-  sh = qmm_shape(W->Npad, W->nkb, M);
+  // The residual epilogue writes a sum-of-squares partial per workgroup: its row tiles, which group the columns of the
+  // next RMSNorm's sum, must not follow M either.
+  sh = qmm_shape(W->Npad, W->nkb, mode == QM_RESID_ACT ? MAX_TOK : M);
   if (rows && sh.KW == 1) sh = qmm_shape_ragged(W->Npad, W->nkb);
   for (const auto& o : c->qmm_shapes) {
     if (o[0] != W->N || o[1] != W->K) continue;
@@ -264,7 +269,7 @@ int launch_qmm_ex(ih_ctx* c, const ih_qmat* W, int expert, const ActBuf& a, int 
   QmmShape sh;
   QmmParams p;
   dim3 grid;
-  IH_TRY(qmm_setup(c, W, expert, M, false, sh, p, grid));
+  IH_TRY(qmm_setup(c, W, expert, M, ep.mode, false, sh, p, grid));
   p.xa = static_cast<const uint4*>(a.frag);
   p.y = ep.y;
   p.ldy = ep.ldy;
@@ -312,7 +317,7 @@ int launch_qmm_rows(ih_ctx* c, const ih_qmat* W, const uint16_t* x, int ldx, int
   QmmShape sh;
   QmmParams p;
   dim3 grid;
-  IH_TRY(qmm_setup(c, W, 0, M, true, sh, p, grid));
+  IH_TRY(qmm_setup(c, W, 0, M, out_mode, true, sh, p, grid));
   // The kernel reads 16-byte pieces of the rows through 32-bit offsets; other rows are copied to aligned scratch first,
   // and so are rows that the output overwrites (some workgroups store while others still read x).
   const uintptr_t x0 = reinterpret_cast<uintptr_t>(x), y0 = reinterpret_cast<uintptr_t>(y);

@@ -369,11 +369,14 @@ def test_rows_do_not_depend_on_the_attention_kernel(ctx, shape, chunk):
         m.free()
 
 
-# MXFP4 experts over 23 K-blocks: the sum over K is split between the waves of a workgroup.
+# MXFP4 experts over 23 K-blocks (the sum over K is split between the waves of a workgroup), and a residual stream of
+# 16384 columns behind a down product whose K no launch shape tiles exactly (23 K-blocks: the row tiles of a workgroup
+# follow the number of rows where no epilogue sums over the columns).
 MOEX23 = dict(MOEX, n_layers=2, hidden=2880, n_experts=32, expert_intermediate=2880, iid_routing=1)
+WIDE = dict(n_layers=1, hidden=16384, n_q_heads=16, n_kv_heads=4, head_dim=64, intermediate=2880, vocab=256)
 
 
-@pytest.mark.parametrize("shape", [MOEX23], ids=["moe-mxfp4-k2880"])
+@pytest.mark.parametrize("shape", [MOEX23, WIDE], ids=["moe-mxfp4-k2880", "hidden-16384"])
 def test_rows_do_not_depend_on_the_launch_shapes(ctx, shape):
     """A row's logits have the same bits in a full block and in every shorter one."""
     d, m, kv = make(ctx, shape)
