@@ -254,7 +254,10 @@ static int qmm_setup(ih_ctx* c, const ih_qmat* W, int expert, int M, int mode, b
   p.nkb = W->nkb;
   p.kmask = 0x000F000Fu;
   p.kbias = 0x43004300u;
-  grid = dim3(W->Npad / (16 * sh.R), sh.ks, sh.ragged && M > 17 ? 2 : 1);
+  // More than 17 of the caller's rows: two token tiles of one product, or two products of 16 rows where the registers
+  // (ragged shapes of 16 waves) or the LDS of two do not fit.
+  const bool two = rows && M > 17 && (sh.ragged || !qmm_fits(2, sh.R, sh.KW, false, sh.kpw));
+  grid = dim3(W->Npad / (16 * sh.R), sh.ks, two ? 2 : 1);
   if (sh.ks > 1) {
     IH_TRY(ensure_qpart(c, size_t(sh.ks) * MAX_TOK * W->Npad * sizeof(float)));
     p.part = c->qpart;

@@ -153,17 +153,21 @@ __device__ __forceinline__ u32x4 frag_order(const u32x4& v) {
 // first two stages; with fewer K-blocks they still end with the first half.
 // XN: the activations are the caller's bf16 rows (16-byte aligned), permuted to the fragment order with four v_perm_b32
 // per MFMA step as they are used; a step past K reads as zero. A separate launch that rearranged them cost more than the
-// product of a small matrix (8 × 4096 × 4096: 3.6 + 4.7 µs). RAG: see QmmShape.
+// product of a small matrix (8 × 4096 × 4096: 3.6 + 4.7 µs). With gridDim.z = 2 (T = 1, more than 17 rows) workgroup z
+// takes rows 16z … as a product of its own, with its own partial sums and arrival counts. RAG: see QmmShape.
 template <int T, int R, int KW, bool X16, int D, int KPW, int MODE, int KPW1 = 0, bool XN = false, bool RAG = false>
 __global__ __launch_bounds__(64 * KW) void qmm_int4_kernel(QmmParams p) {
-  if constexpr (RAG) {
-    // Rows 16·z … of a launch of more than 17 rows (two token tiles' registers do not fit 16 waves).
-    const int z = int(blockIdx.z);
-    p.xa = reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(p.xa) + size_t(16 * z) * p.ldx);
-    p.y = static_cast<char*>(p.y) + size_t(16 * z) * p.ldy * (MODE == QM_BF16 ? 2 : 4);
-    if (gridDim.z > 1) p.M = min(16, p.M - 16 * z);
-    p.part += size_t(16 * z) * p.Npad;
-    p.ctr += z * int(gridDim.x);
+  if constexpr (XN && T == 1 && !X16) {
+    if (gridDim.z > 1) {
+      const int z = int(blockIdx.z);
+      p.xa = reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(p.xa) + size_t(16 * z) * p.ldx);
+      p.y = static_cast<char*>(p.y) + size_t(16 * z) * p.ldy * (MODE == QM_BF16 ? 2 : 4);
+      p.M = min(16, p.M - 16 * z);
+      if (gridDim.y > 1) {
+        p.part += size_t(16 * z) * p.Npad;
+        p.ctr += z * int(gridDim.x);
+      }
+    }
   }
   static_assert(KPW % D == 0 && KPW1 % D == 0, "the ring depth divides the K-blocks of a wave");
   // The wave index is uniform: readfirstlane keeps it (and everything derived from it) in scalar registers.
@@ -517,8 +521,9 @@ __global__ __launch_bounds__(64 * KW) void qmm_int4_kernel(QmmParams p) {
 struct QmmShape { int R, KW, D, kpw, ks, kpw1 = 0, ragged = 0; };
 constexpr int qmm_ring_depth(int kpw) { return kpw % 2 == 0 ? 2 : kpw <= 3 ? kpw : 1; }
 
-template <int T, int R, int KW, bool X16, int KPW>
-constexpr bool qmm_fits() {
+// Whether a shape's LDS fits with T token tiles (and token 16 on its own): only those are instantiated. Two tiles of
+// (7, 8, 6) do not: the caller's rows past 17 go as two groups of 16 there (qmm_setup).
+constexpr bool qmm_fits(int T, int R, int KW, bool X16, int KPW) {
   return 4 * KW * (R * T * 256 + (X16 ? R * 16 : 0)) + 4 * MAX_TOK * (2 * R + 1) + R * KW * KPW * 128 +
              (X16 ? KW * KPW * 512 : 0) <= 128 * 1024;
 }
@@ -528,7 +533,7 @@ constexpr bool qmm_fits() {
 template <int T, bool X16, int MODE, bool XN = false>
 static bool qmm_dispatch_mode(const TimedLaunch& tl, QmmShape sh, dim3 grid, hipStream_t st, const QmmParams& p) {
 #define IH_QMM_CASE(R_, KW_, KPW_)                                                                          \
-  if constexpr (qmm_fits<T, R_, KW_, X16, KPW_>()) {                                                        \
+  if constexpr (qmm_fits(T, R_, KW_, X16, KPW_)) {                                                        \
     if (sh.R == R_ && sh.KW == KW_ && sh.kpw == KPW_ && sh.kpw1 == 0 && !sh.ragged) {                                     \
       tlaunch(tl, qmm_int4_kernel<T, R_, KW_, X16, qmm_ring_depth(KPW_), KPW_, MODE, 0, XN>, grid,            \
               dim3(64 * KW_), 0, st, p);                                                                                       \
@@ -544,7 +549,7 @@ static bool qmm_dispatch_mode(const TimedLaunch& tl, QmmShape sh, dim3 grid, hip
 #undef IH_QMM_CASE
   // Asymmetric K split (KPW for the first half of the waves, KPW1 for the second): gate|up at two waves per SIMD.
 #define IH_QMM_CASE1(R_, KW_, KPW_, KPW1_)                                                                       \
-  if constexpr (qmm_fits<T, R_, KW_, X16, KPW_>()) {                                                        \
+  if constexpr (qmm_fits(T, R_, KW_, X16, KPW_)) {                                                        \
     if (sh.R == R_ && sh.KW == KW_ && sh.kpw == KPW_ && sh.kpw1 == KPW1_) {                                \
       tlaunch(tl, qmm_int4_kernel<T, R_, KW_, X16, 2, KPW_, MODE, KPW1_, XN>, grid, dim3(64 * KW_), 0, st, p);   \
       return true;                                                                                          \
@@ -554,7 +559,7 @@ static bool qmm_dispatch_mode(const TimedLaunch& tl, QmmShape sh, dim3 grid, hip
 #undef IH_QMM_CASE1
   if constexpr (XN && T == 1) {
 #define IH_QMM_CASER(R_, KW_, KPW_)                                                                                 \
-  if constexpr (qmm_fits<T, R_, KW_, X16, KPW_>()) {                                                                \
+  if constexpr (qmm_fits(T, R_, KW_, X16, KPW_)) {                                                                \
     if (sh.ragged && sh.R == R_ && sh.KW == KW_ && sh.kpw == KPW_) {                                                \
       tlaunch(tl, qmm_int4_kernel<T, R_, KW_, X16, qmm_ring_depth(KPW_), KPW_, MODE, 0, true, true>, grid,          \
               dim3(64 * KW_), 0, st, p);                                                                            \
@@ -569,7 +574,7 @@ static bool qmm_dispatch_mode(const TimedLaunch& tl, QmmShape sh, dim3 grid, hip
   return false;  // not an instantiated shape
 }
 
-// qmm_rows.hip: the launch on bf16 rows.
+// qmm_rows.hip: the launch on bf16 rows (more than 17: two token tiles, or grid.z = 2 groups of 16).
 bool qmm_rows_dispatch(const TimedLaunch& tl, QmmShape sh, dim3 grid, hipStream_t st, const QmmParams& p, int M,
                        int mode);
 

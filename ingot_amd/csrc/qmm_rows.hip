@@ -16,7 +16,7 @@ static bool by_mode(const TimedLaunch& tl, QmmShape sh, dim3 grid, hipStream_t s
 
 bool qmm_rows_dispatch(const TimedLaunch& tl, QmmShape sh, dim3 grid, hipStream_t st, const QmmParams& p, int M,
                        int mode) {
-  if (M > 17 && !sh.ragged) return by_mode<2, false>(tl, sh, grid, st, p, mode);
+  if (M > 17 && grid.z == 1) return by_mode<2, false>(tl, sh, grid, st, p, mode);
   if (M == 17) return by_mode<1, true>(tl, sh, grid, st, p, mode);
   return by_mode<1, false>(tl, sh, grid, st, p, mode);
 }

@@ -229,3 +229,24 @@ def test_qmm_output_over_its_own_rows(ctx, mode):
     finally:
         W.free()
     assert np.array_equal(got.view(np.uint8), want.view(np.uint8))
+
+
+@pytest.mark.parametrize("N,K", [x for x in CFG1_SHAPES if x != (151936, 4096)] + TILED)
+def test_qmm_more_rows_than_a_block(ctx, N, K):
+    """18 … 32 rows through every launch shape: the first 17 rows have the bits of the 17-row product, the others those
+    of a product of their own."""
+    g = rng(N + K + 1)
+    w = g.integers(0, 2**32, size=(N, K // 8), dtype=np.uint32)
+    s = oracle.f32_to_bf16(np.abs(g.normal(0, 0.02, size=(N, K // 64))).astype(np.float32))
+    xb, _ = bf16_normal(g, (32, K))
+    W = QMat.int4(ctx, w, s, oracle.f32_to_bf16(-8.0 * oracle.bf16_to_f32(s)))
+    try:
+        want = np.concatenate([run_qmm(ctx, W, xb[:17].copy(), 17), run_qmm(ctx, W, xb[17:].copy(), 15)])
+        assert np.isfinite(want).all()
+        for m in (18, 32):
+            got = run_qmm(ctx, W, xb[:m].copy(), m)
+            assert np.array_equal(got.view(np.uint32), want[:m].view(np.uint32)), m
+            got = run_qmm(ctx, W, xb[:m].copy(), m, out_mode=2)
+            assert np.array_equal(got, oracle.f32_to_bf16(want[:m])), m
+    finally:
+        W.free()
