@@ -282,7 +282,8 @@ __device__ __forceinline__ void attn_step(TileState<HD>& st, const f16x8 (&qf)[H
   mx = row_max4(mx);
   // The reference of a row's exponents is its first visible step's max, moved only when a later max passes it by RAISE
   // in log2 units: most steps then leave O as it is (a new max somewhere among 16 rows would rescale it nearly every
-  // step). Weights stay ≤ 2^RAISE.
+  // step). Weights stay ≤ 2^RAISE; times a V scale above 65504 / 2^RAISE one may pass the range of the fp16 product, and
+  // the reduction then takes the row's split without it (split_in_fp32).
   const bool raise = mx * sc > fmaf(st.mrun, sc, RAISE) || st.mrun == -INFINITY;
   const float mnew = raise ? mx : st.mrun;
   const float alpha = raise && mnew != -INFINITY ? __builtin_amdgcn_exp2f((st.mrun - mnew) * sc) : 1.f;
@@ -329,6 +330,13 @@ __device__ __forceinline__ void attn_merge(const AttnArgs& a, TileState<HD>& st,
     float l = st.lsum;
     l += lane_xor<16>(l);
     l += lane_xor<32>(l);
+    // A weight that overflowed leaves no dim of its row finite: any one tells. The NaN sum reaches the reduction; the
+    // partial itself stays finite, for lanes of the reduction that read it in an idle place.
+    if (!(fabsf(st.o[0][0]) < INFINITY)) {
+      l = NAN;
+#pragma unroll
+      for (int dt = 0; dt < NDT; ++dt) st.o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
     if (qd == 0) sml[cls][lt][j] = make_float2(st.mrun, l);
   }
   __syncthreads();
@@ -611,6 +619,60 @@ __global__ __launch_bounds__(64 * NCLS * FEW) void attn_few_kernel(AttnArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------------------------------
+// One row's split again, by a whole wave: softmax over its visible keys in fp32 with weights of at most 1, for rows whose
+// weights times V scales passed fp16 in the kernels above (their limit would otherwise be a sixteenth of what the cache
+// holds: values of 5e5). O / l in fp16 as those write it, the lane's eight dims 8dg … in raw; returns (reference, sum).
+// A test of the scales in every step instead, or a second pass inside those kernels, cost 0.5 to 1 % of a step's time;
+// this costs nothing measurable (dense, 17 rows at 8K: 2238 µs a step with and without).
+template <int HD>
+__device__ __forceinline__ float2 split_in_fp32(const AttnArgs& a, int kvh, int m, int sidx, int lane, int dg, uint4& raw) {
+  constexpr int NE = HD / 64;
+  const AttnPos ap = attn_pos(a);
+  const SplitKeys sk = split_keys(a, ap, sidx);
+  const int row = ap.P + m / a.G;
+  const int k0 = max(sk.kbase, a.window > 0 ? row - a.window + 1 : 0), k1 = min(sk.k1, row + 1);
+  float q[NE], o[NE], M = -INFINITY, l = 0.f;
+#pragma unroll
+  for (int e = 0; e < NE; ++e) {
+    q[e] = __half2float(a.q[(size_t(kvh) * a.Qpad + m) * HD + lane + 64 * e]);
+    o[e] = 0.f;
+  }
+  for (int key = k0; key < k1; ++key) {
+    const int slot = a.ring ? key % a.ring : key;
+    const size_t hs = size_t(kvh) * a.vld + slot;
+    float s = 0.f;
+#pragma unroll
+    for (int e = 0; e < NE; ++e) s = fmaf(q[e], float(a.kc[k_index(kvh, slot, lane + 64 * e, HD, a.vld)]) - 128.f, s);
+    s += lane_xor<32>(s);
+    s += lane_xor<16>(s);
+    s += lane_xor<8>(s);
+    s += lane_xor<4>(s);
+    s += lane_xor<2>(s);
+    s += lane_xor<1>(s);
+    s *= __half2float(a.ks[hs]) * a.scale_log2;
+    const float Mn = fmaxf(M, s), c = M == -INFINITY ? 0.f : exp2f(M - Mn), p = Mn == -INFINITY ? 0.f : exp2f(s - Mn);
+    const float w = p * __half2float(a.vs[hs]);
+    l = fmaf(l, c, p);
+#pragma unroll
+    for (int e = 0; e < NE; ++e)
+      o[e] = fmaf(w, float(a.vc[v_index(kvh, slot, lane + 64 * e, HD, a.vld)]) - 128.f, o[e] * c);
+    M = Mn;
+  }
+  unsigned h[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int d = 8 * dg + i;
+    float v = __shfl(o[0], d & 63);
+    if constexpr (NE == 2) {
+      const float v1 = __shfl(o[1], d & 63);
+      v = d >= 64 ? v1 : v;
+    }
+    h[i] = __half_as_ushort(__float2half_rn(l > 0.f ? v / l : 0.f));
+  }
+  raw = make_uint4(h[0] | h[1] << 16, h[2] | h[3] << 16, h[4] | h[5] << 16, h[6] | h[7] << 16);
+  return make_float2(M, l);
+}
+
 // Reduction of the splits (vattn_reduce, verify_attn.metal:149-192): M = max over splits (and the sink), L = Σ e^(m−M)·l
 // (+ e^(sink−M)), o = Σ e^(m−M)·l·ō / L with ō = O/l the split's normalised partial; written into the o_proj
 // activation layout (column h·HD + d). One wave per (row, q head): lane = (split group sg, 8-dim group dg); a lane
@@ -683,6 +745,32 @@ __global__ __launch_bounds__(64) void attn_reduce_kernel(AttnArgs a, uint4* __re
   if constexpr (DG <= 8) merge(std::integral_constant<int, 8>{});
   merge(std::integral_constant<int, 16>{});
   merge(std::integral_constant<int, 32>{});
+  if (__builtin_expect(__any(L != L), 0)) {
+    // Some split's weights overflowed: the row once more, that split in fp32, the splits in order. The arguments are read
+    // again here from the kernel's argument segment, which they head: hoisted, their loads cost every launch 0.2 µs.
+    const AttnArgs* ac = (const AttnArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(ac));
+    M = -INFINITY;
+    L = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = 0.f;
+    for (int s = 0; s < nsplit; ++s) {
+      const size_t idx = (size_t(kvh) * a.nsplit + s) * a.Qpad + m;
+      float2 f = a.ml[idx];
+      uint4 raw = *reinterpret_cast<const uint4*>(a.opart + idx * HD + 8 * dg);
+      if (f.y != f.y) f = split_in_fp32<HD>(*ac, kvh, m, s, lane, dg, raw);  // uniform
+      if (f.x == -INFINITY) continue;
+      const float Mn = fmaxf(M, f.x), c = M == -INFINITY ? 0.f : exp2f(M - Mn), w = exp2f(f.x - Mn) * f.y;
+      const unsigned rw[4] = {raw.x, raw.y, raw.z, raw.w};
+      L = L * c + w;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float2 h = __half22float2(__builtin_bit_cast(__half2, rw[e >> 1]));
+        o[e] = o[e] * c + w * ((e & 1) ? h.y : h.x);
+      }
+      M = Mn;
+    }
+  }
   if (sg != 0) return;
   // The sink is a last split with weight e^(sink−M) and no value, merged after the splits' tree so that its place
   // does not depend on which split a window starts in (the same bits for a row whatever the block's P).

@@ -390,3 +390,66 @@ def test_rows_do_not_depend_on_the_launch_shapes(ctx, shape):
     finally:
         kv.free()
         m.free()
+
+
+def _scale_tensor(path, name, factor):
+    """Multiplies a bf16 tensor of a safetensors file in place."""
+    import json
+    import struct
+
+    raw = bytearray(path.read_bytes())
+    n = struct.unpack("<Q", raw[:8])[0]
+    a, b = json.loads(raw[8: 8 + n])[name]["data_offsets"]
+    v = np.frombuffer(bytes(raw[8 + n + a: 8 + n + b]), np.uint16)
+    raw[8 + n + a: 8 + n + b] = oracle.f32_to_bf16(oracle.bf16_to_f32(v) * np.float32(factor)).tobytes()
+    path.write_bytes(raw)
+
+
+# One layer of 128-dim heads, and one of 64-dim heads with sinks and a ring of 4096 keys.
+RANGE = dict(SMALL, n_layers=1)
+RANGE64 = dict(n_layers=1, hidden=192, n_q_heads=8, n_kv_heads=2, head_dim=64, intermediate=0, vocab=777, n_experts=8,
+               top_k=4, expert_intermediate=96, expert_format=1, act=1, sinks=1, sliding_window=4096, router_int4=1)
+
+
+@pytest.mark.parametrize("shape,family,factor", [(RANGE, "", 1.25), (RANGE64, "gpt_oss", 1.5625)],
+                         ids=["hd128", "hd64-ring-sinks"])
+def test_attention_weights_times_the_largest_value_scales(ctx, tmp_path, shape, family, factor):
+    """Values near the top of the cache's range (an int8 value's fp16 scale goes up to 65504; 4094 · 16 is the first that
+    a weight above 1 could take past fp16): an attention weight is multiplied by that scale and rounded to fp16, and must
+    not overflow there. v_proj × 2^16 with o_proj × 2^-16 is the model with 2^4 and 2^-4: scales and products follow
+    exactly, so only roundings of weights may differ. The embedding and v_proj are centred (codes − 7.5), so that the
+    average over thousands of keys stays below the values (in 64 bits, with these factors: averages up to 49000, weights
+    of up to 2^4 of a first step's maximum times their scales up to 83800)."""
+    import sys
+    from pathlib import Path
+    sys.path.insert(0, str(Path(__file__).resolve().parent / "golden"))
+    from make_mlx_checkpoint import write_checkpoint
+
+    got = {}
+    for k in (4, 16):
+        out = write_checkpoint(tmp_path / str(k), shape, seed=7, family=family)
+        f = out / "model.safetensors"
+        attn = "model.layers.0.self_attn."
+        _scale_tensor(f, "model.embed_tokens.biases", 15 / 16)
+        _scale_tensor(f, attn + "v_proj.biases", 15 / 16)
+        for part in ("scales", "biases"):
+            _scale_tensor(f, attn + f"q_proj.{part}", 0.5)
+            _scale_tensor(f, attn + f"v_proj.{part}", factor * 2.0 ** k)
+            _scale_tensor(f, attn + f"o_proj.{part}", 2.0 ** -k)
+        m = Model.load_mlx(ctx, out)
+        kv = KVCache(m, 8192, 8192)  # one split: its partial is the average over every key
+        try:
+            toks = np.random.default_rng(5).integers(0, shape["vocab"], size=8160).astype(np.uint32)
+            for i in range(0, 8160 - 17, 17):
+                kv.verify(toks[i: i + 17])
+                kv.commit(17)
+            _, got[k] = kv.verify(toks[-17:], want_logits=True)
+            for n in (1, 4, 12):
+                _, part = kv.verify(toks[-17:][:n], want_logits=True)
+                assert np.array_equal(part.view(np.uint32), got[k][:n].view(np.uint32)), (k, n)
+        finally:
+            kv.free()
+            m.free()
+    scale = np.abs(got[4]).max()
+    assert np.isfinite(got[16]).all()
+    assert np.abs(got[16] - got[4]).max() <= 0.02 + 0.01 * scale
