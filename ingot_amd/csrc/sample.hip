@@ -93,17 +93,19 @@ __device__ __forceinline__ void lse_batch(const float (&c)[N], const bool (&ok)[
 //      smallest of the 32 second bests is a value that at least 64 logits of the row reach.
 //   2. topk64_collect_kernel, the same workgroups: the chunk's logits that reach it, in any order, to the chunk's own
 //      slots (≈ 170 of 151936 per row for independent logits; one list per row behind a global counter took 38 µs).
-//   3. topk64_final_kernel, one workgroup per row: the candidates sorted. A row with a chunk that has more candidates
-//      than slots (many equal logits) is scanned instead, each wave keeping its running best 64.
-// Values below −FLT_MAX and NaN are never candidates; missing entries are (−FLT_MAX, NO_ID).
+//   3. topk64_final_kernel, one workgroup per row: the candidates sorted.
+// A chunk with more candidates than slots (many logits equal to the bound, e.g. a vocabulary masked with one finite value)
+// hands on those above the bound and the first 64 equal to it; one with more than 64 above it, its best 64. Values below
+// −FLT_MAX and NaN are never candidates; missing entries are (−FLT_MAX, NO_ID).
 // A 17 × 151936 round: bound 6.9, collect 4.3, final 7.9 µs, against 28 + 9 for running best-64 lists per chunk and their
-// merge, whose sorting networks were one long dependency chain per wave.
+// merge, whose sorting networks were one long dependency chain per wave. With all but 40 logits of a row at −1e9: 23.4 µs
+// (81 where one workgroup scanned such a row, 23.0 by the lists).
 constexpr int CCAP = 128;        // candidates kept per chunk (sorted logits: one block of 64)
 struct TopScratch {
   float* thr;    // [rows][SPG] second best of each chunk
   float2* pz;    // [rows][SPG] (max, Σ exp)
-  unsigned* cnt; // [rows][SPG] candidates found
-  uint2* cand;   // [rows][SPG][CCAP] (value bits, id)
+  unsigned* cnt; // [rows][SPG] candidates; crowded: above the bound | equal << 8 | equal in the first block << 16
+  uint2* cand;   // [rows][SPG][CCAP] (value bits, id); crowded: above the bound from 0, equal to it from SK
 };
 
 __global__ __launch_bounds__(SPT) void topk64_bound_kernel(const float* __restrict__ x, int ldx, int V, float temp,
@@ -172,6 +174,21 @@ __global__ __launch_bounds__(SPT) void topk64_bound_kernel(const float* __restri
   t.pz[row * SPG + g] = make_float2(M, Z);
 }
 
+// The NW lists of a workgroup (one per wave, descending in v/id) merged into wave 0's.
+template <int NW>
+__device__ __forceinline__ void merge_waves(float& v, uint32_t& id, float (*sv)[SK], uint32_t (*si)[SK], int wave,
+                                            int lane) {
+#pragma unroll
+  for (int n = NW / 2; n >= 1; n >>= 1) {  // waves n … 2n − 1 hand theirs to waves 0 … n − 1
+    if (wave >= n && wave < 2 * n) {
+      sv[wave][lane] = v;
+      si[wave][lane] = id;
+    }
+    __syncthreads();
+    if (wave < n) merge64(v, id, sv[wave + n][lane], si[wave + n][lane], lane);
+  }
+}
+
 __global__ __launch_bounds__(SPT) void topk64_collect_kernel(const float* __restrict__ x, int ldx, int V, TopScratch t) {
   constexpr int NB = 8;
   __shared__ unsigned count;
@@ -204,24 +221,103 @@ __global__ __launch_bounds__(SPT) void topk64_collect_kernel(const float* __rest
     }
   }
   __syncthreads();
-  if (threadIdx.x == 0) t.cnt[row * SPG + g] = count;
-}
-
-// The workgroup's lists (one per wave, descending in v/id) merged into wave 0's.
-constexpr int FT = 512;  // threads of the final kernel
-__device__ __forceinline__ void merge_waves(float& v, uint32_t& id, float (*sv)[SK], uint32_t (*si)[SK], int wave,
-                                            int lane) {
-#pragma unroll
-  for (int n = FT / 128; n >= 1; n >>= 1) {  // waves n … 2n − 1 hand theirs to waves 0 … n − 1
-    if (wave >= n && wave < 2 * n) {
-      sv[wave][lane] = v;
-      si[wave][lane] = id;
-    }
-    __syncthreads();
-    if (wave < n) merge64(v, id, sv[wave + n][lane], si[wave + n][lane], lane);
+  const unsigned n = count;  // uniform
+  if (n <= unsigned(CCAP)) {
+    if (threadIdx.x == 0) t.cnt[row * SPG + g] = n;
+    return;
   }
+  // Too many: the values above the bound to slots 0 …, of those equal to it the first 64 in order to slots SK … (block j of
+  // the chunk is wave j mod 4's).
+  constexpr int NW = SPT / 64;
+  __shared__ unsigned above, eqb[NW * NB];
+  unsigned taken = 0, first = 0;  // uniform: equal values so far (to 64), those of the chunk's first block
+  if (threadIdx.x == 0) above = 0u;
+  __syncthreads();
+  for (int b0 = 64 * g; b0 < V; b0 += STRIDE * NB) {  // uniform over the workgroup
+    const int base = b0 + 64 * SPG * wave;
+    float c[NB];
+#pragma unroll
+    for (int u = 0; u < NB; ++u) c[u] = xr[min(base + STRIDE * u + lane, V - 1)];
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
+      const int i = base + STRIDE * u + lane;
+      const unsigned long long mask = __ballot(i < V && c[u] > thr);
+      if (mask) {
+        unsigned at = 0;
+        if (lane == 0) at = atomicAdd(&above, unsigned(__popcll(mask)));
+        at = __builtin_amdgcn_readfirstlane(at) + unsigned(__popcll(mask & ((1ull << lane) - 1ull)));
+        if ((mask >> lane & 1ull) && at < SK) cand[at] = make_uint2(__float_as_uint(c[u]), uint32_t(i));
+      }
+      const unsigned long long eq = __ballot(i < V && c[u] == thr);
+      if (lane == 0) eqb[NW * u + wave] = unsigned(__popcll(eq));
+    }
+    if (taken >= SK) continue;
+    __syncthreads();
+    unsigned e = lane < NW * NB ? eqb[lane] : 0u, sum = e;
+#pragma unroll
+    for (int d = 1; d < NW * NB; d <<= 1) {
+      const unsigned o = __shfl_up(sum, d);
+      if (lane >= d) sum += o;
+    }
+    if (b0 == 64 * g) first = min(__builtin_amdgcn_readlane(e, 0), unsigned(SK));
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
+      const int j = NW * u + wave, i = base + STRIDE * u + lane;
+      const unsigned before = taken + __builtin_amdgcn_readlane(sum, j) - __builtin_amdgcn_readlane(e, j);
+      if (before >= SK) continue;
+      const unsigned long long eq = __ballot(i < V && c[u] == thr);
+      const unsigned at = before + unsigned(__popcll(eq & ((1ull << lane) - 1ull)));
+      if ((eq >> lane & 1ull) && at < SK) cand[SK + at] = make_uint2(__float_as_uint(c[u]), uint32_t(i));
+    }
+    taken = min(taken + __builtin_amdgcn_readlane(sum, NW * NB - 1), unsigned(SK));
+    __syncthreads();
+  }
+  __syncthreads();
+  const unsigned na = above;  // uniform
+  if (na <= SK) {
+    if (threadIdx.x == 0) t.cnt[row * SPG + g] = na | taken << 8 | first << 16;
+    return;
+  }
+  // More than 64 above the bound as well: the chunk's best 64, by a running list per wave. A block enters its wave's list
+  // only if one of its values beats the list's last entry (a lane's batch in LDS: a register file has no index).
+  __shared__ float sv[NW][SK];
+  __shared__ uint32_t si[NW][SK];
+  __shared__ float batch[NB][SPT];
+  float v = -FLT_MAX;
+  uint32_t id = NO_ID;
+  auto enters = [&](float b, uint32_t bid) {
+    const float tv = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+    const uint32_t ti = uint32_t(__builtin_amdgcn_readlane(int(id), 63));
+    return __any(tk_better(b, bid, tv, ti));
+  };
+  for (int base = 64 * (g + SPG * wave); base < V; base += STRIDE * NB) {
+    float c[NB];
+#pragma unroll
+    for (int u = 0; u < NB; ++u) c[u] = xr[min(base + STRIDE * u + lane, V - 1)];
+    unsigned need = 0;  // uniform: the batch's blocks that may enter
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
+      const int i = base + STRIDE * u + lane;
+      c[u] = i < V && c[u] > thr ? c[u] : -INFINITY;
+      batch[u][threadIdx.x] = c[u];
+      need |= enters(c[u], uint32_t(i)) ? 1u << u : 0u;
+    }
+    for (; need; need &= need - 1) {
+      const int u = __builtin_ctz(need);
+      float b = batch[u][threadIdx.x];
+      uint32_t bid = b == -INFINITY ? NO_ID : uint32_t(base + STRIDE * u + lane);
+      b = b == -INFINITY ? -FLT_MAX : b;
+      if (!enters(b, bid)) continue;
+      sort64(b, bid, lane);
+      merge64(v, id, b, bid, lane);
+    }
+  }
+  merge_waves<NW>(v, id, sv, si, wave, lane);
+  if (wave == 0) cand[lane] = make_uint2(__float_as_uint(v), id);
+  if (threadIdx.x == 0) t.cnt[row * SPG + g] = unsigned(SK);
 }
 
+constexpr int FT = 512;  // threads of the final kernel
 __global__ __launch_bounds__(FT) void topk64_final_kernel(const float* __restrict__ x, int ldx, int V, float temp,
                                                           TopScratch t, uint32_t* __restrict__ idx,
                                                           float* __restrict__ val, float* __restrict__ z) {
@@ -229,62 +325,49 @@ __global__ __launch_bounds__(FT) void topk64_final_kernel(const float* __restric
   __shared__ uint32_t si[FT / 64][SK];
   __shared__ uint2 list[SPG * CCAP];
   const int row = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  // The chunks' counts, one per lane of the lower half, and where each chunk's candidates start in the row's list.
-  const unsigned cn = lane < SPG ? t.cnt[row * SPG + lane] : 0u;
-  const bool fits = !__any(cn > unsigned(CCAP));
-  unsigned at = fits ? cn : 0u;
+  // The chunks' counts, one per lane of the lower half: candidates; in crowded chunks those above the bound, those equal to
+  // it and how many of these lie in the chunk's first block. The first blocks of all chunks are the row's first logits, so
+  // where they hold 64 equal values no others are needed. Then where each chunk's candidates start in the row's list.
+  const unsigned cw = lane < SPG ? t.cnt[row * SPG + lane] : 0u, cn = cw & 255u, e0 = cw >> 16;
+  auto scan = [&](unsigned x) {
 #pragma unroll
-  for (int d = 1; d < SPG; d <<= 1) {
-    const unsigned o = __shfl_up(at, d);
-    if (lane >= d) at += o;
-  }
-  const unsigned n = __builtin_amdgcn_readlane(at, SPG - 1);
-  if (fits) {
-    for (int g = wave; g < SPG; g += FT / 64) {
-      const unsigned cg = __builtin_amdgcn_readlane(cn, g), ag = __builtin_amdgcn_readlane(at, g) - cg;
-      for (unsigned k = lane; k < cg; k += 64) list[ag + k] = t.cand[(size_t(row) * SPG + g) * CCAP + k];
+    for (int d = 1; d < SPG; d <<= 1) {
+      const unsigned o = __shfl_up(x, d);
+      if (lane >= d) x += o;
     }
+    return x;
+  };
+  unsigned eq = cw >> 8 & 255u;
+  if (__any(eq != 0u)) {
+    const unsigned upto = scan(e0);
+    if (__builtin_amdgcn_readlane(upto, SPG - 1) >= SK) eq = min(e0, unsigned(max(0, SK - int(upto - e0))));
+  }
+  const unsigned at = scan(cn + eq), n = __builtin_amdgcn_readlane(at, SPG - 1);
+  for (int g = wave; g < SPG; g += FT / 64) {
+    const unsigned cg = __builtin_amdgcn_readlane(cn, g), eg = __builtin_amdgcn_readlane(eq, g);
+    const unsigned ag = __builtin_amdgcn_readlane(at, g) - cg - eg;
+    const uint2* cand = t.cand + (size_t(row) * SPG + g) * CCAP;
+    for (unsigned k = lane; k < cg + eg; k += 64) list[ag + k] = cand[k < cg ? k : SK + k - cg];
   }
   __syncthreads();
   const float it = 1.0f / temp;
   float v = -FLT_MAX;
   uint32_t id = NO_ID;
-  // A batch of 64 values (one per lane) into the wave's list.
-  auto take = [&](float c, uint32_t cid) {
+  bool first = true;
+  for (unsigned b = 64 * wave; b < n; b += FT) {  // a batch of 64 candidates, one per lane, into the wave's list
+    const uint2 w = b + lane < n ? list[b + lane] : make_uint2(__float_as_uint(-FLT_MAX), NO_ID);
+    float c = __uint_as_float(w.x);
+    uint32_t cid = w.y;
     sort64(c, cid, lane);
-    merge64(v, id, c, cid, lane);
-  };
-  if (fits) {
-    bool first = true;
-    for (unsigned b = 64 * wave; b < n; b += FT) {
-      const uint2 w = b + lane < n ? list[b + lane] : make_uint2(__float_as_uint(-FLT_MAX), NO_ID);
-      float c = __uint_as_float(w.x);
-      uint32_t cid = w.y;
-      if (first) {
-        sort64(c, cid, lane);
-        v = c;
-        id = cid;
-        first = false;
-      } else {
-        take(c, cid);
-      }
-    }
-  } else {
-    // More candidates than fit: the waves scan the row, a batch entering a wave's list only if one of its values beats
-    // the list's last entry.
-    const float* xr = x + size_t(row) * ldx;
-    for (int base = 64 * wave; base < V; base += FT) {
-      const int i = base + lane;
-      float c = xr[min(i, V - 1)];
-      const bool ok = i < V && c == c && c >= -FLT_MAX;
-      const uint32_t cid = ok ? uint32_t(i) : NO_ID;
-      if (!ok) c = -FLT_MAX;
-      const float tv = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
-      const uint32_t ti = uint32_t(__builtin_amdgcn_readlane(int(id), 63));
-      if (__any(tk_better(c, cid, tv, ti))) take(c, cid);
+    if (first) {
+      v = c;
+      id = cid;
+      first = false;
+    } else {
+      merge64(v, id, c, cid, lane);
     }
   }
-  merge_waves(v, id, sv, si, wave, lane);
+  merge_waves<FT / 64>(v, id, sv, si, wave, lane);
   if (wave != 0) return;
   idx[size_t(row) * SK + lane] = id;
   val[size_t(row) * SK + lane] = v;

@@ -44,9 +44,8 @@ def test_topk64_matches_oracle(ctx, rows, V):
 
 @pytest.mark.parametrize("order", ["ascending", "descending", "sawtooth"])
 def test_topk64_buffer_paths_match_oracle(ctx, order):
-    """Orders that drive the chunk kernel's candidate buffer to its extremes: ascending logits make every element beat
-    the running 64th best (a flush per 64 elements), descending ones admit only the first 64 of each wave, a sawtooth
-    mixes both with ties across the teeth."""
+    """Orders that drive the selection to its extremes: ascending and descending logits put the 64 best into one or two
+    blocks of 64 and every other chunk's second best far below them, a sawtooth mixes ties across the teeth."""
     rows, V = 5, 151936
     base = np.arange(V, dtype=np.float32)
     x = {"ascending": base / 1000.0, "descending": -base / 1000.0, "sawtooth": np.float32(0.25) * (base % 997)}[order]
@@ -65,7 +64,7 @@ def test_topk64_buffer_paths_match_oracle(ctx, order):
 @pytest.mark.parametrize("V", [1, 63, 64, 65, 1984, 2047, 2049, 4095, 8192, 50257])
 def test_topk64_sparse_and_crowded_rows(ctx, V):
     """Rows at the edges of the two-pass selection: fewer than 64 finite logits, every logit equal (all of them reach the
-    bound: past 4096 the row is scanned), two values in blocks, one chunk masked out, all NaN, V below and above one
+    bound: past 4096 the chunks are crowded), two values in blocks, one chunk masked out, all NaN, V below and above one
     64-logit block per chunk; rows apart by more than V."""
     g = np.random.default_rng(V)
     rows, ld = 7, V + 5
@@ -88,6 +87,34 @@ def test_topk64_sparse_and_crowded_rows(ctx, V):
     assert np.array_equal(gv, ov)
     assert np.array_equal(gz[:, 0], oz[:, 0])
     assert np.allclose(gz[:, 1], oz[:, 1], rtol=2e-5, equal_nan=True)
+
+
+@pytest.mark.parametrize("V,mask", [(151936, -1e9), (151936, -65504.0), (50257, -3.4028234663852886e38), (4160, -1e9),
+                                    (4096, -1e9), (32000, 5.0)])
+def test_topk64_many_equal_logits(ctx, V, mask):
+    """Rows whose bound is a value that many logits share (a vocabulary masked with a finite value; a plateau above the
+    other logits): chunks with more candidates than slots, beside chunks with few, ties across chunks by the lower id.
+    The candidates are the finite logits in a stable descending order (the oracle leaves out −FLT_MAX itself)."""
+    g = np.random.default_rng(V)
+    rows = 8
+    x = (g.normal(size=(rows, V)) * 3).astype(np.float32)
+    for r, live in enumerate((0, 1, 40, 63, 64, 200, V // 2)):
+        keep = np.zeros(V, bool)
+        keep[g.choice(V, size=live, replace=False)] = True
+        x[r, ~keep] = mask
+    x[7, 64 * 32 * 20: 64 * 32 * 20 + 64] = 40.0  # one block alone
+    x[7, : V // 64 * 64].reshape(-1, 64)[3::32] = mask  # one chunk masked
+    x[6, ::7] = np.nan
+    x[5, ::3] = -np.inf
+    gi, gv, gz = gpu_topk(ctx, x, 0.8)
+    _, _, oz = oracle.topk64(x, 0.8)
+    for r in range(rows):
+        ids = np.flatnonzero(np.isfinite(x[r]))
+        ids = ids[np.argsort(-x[r, ids].astype(np.float64), kind="stable")][:64]
+        assert np.array_equal(gi[r], ids.astype(np.uint32)), r
+        assert np.array_equal(gv[r], x[r, ids]), r
+    assert np.array_equal(gz[:, 0], oz[:, 0])
+    assert np.allclose(gz[:, 1], oz[:, 1], rtol=2e-5)
 
 
 def test_accept_sample_matches_oracle(ctx):
