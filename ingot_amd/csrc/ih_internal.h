@@ -133,7 +133,7 @@ struct ih_ctx {
   std::vector<hipEvent_t> ev_pool;
   size_t ev_used = 0;
   hipStream_t stream = nullptr;
-  // Argmax scratch: chunk maxima and arrival counts of amax_rows rows.
+  // Argmax scratch of amax_rows rows (AmaxRow, rowops.hip).
   void* amax = nullptr;
   int amax_rows = 0;
   // Scratch of the copy-lookup reduction (ensure_part).

@@ -174,32 +174,40 @@ __global__ __launch_bounds__(256) void argmax_chunk_kernel(const float* __restri
   if (threadIdx.x == 0) part[blockIdx.x * ARGMAX_CHUNKS + blockIdx.y] = make_float2(b, __uint_as_float(ix));
 }
 
+// A row's scratch: the chunks' maxima and the arrival count, each in a memory line of its own. (The counts of 17 rows side
+// by side made all 272 arrivals of a launch queue on one line: 17 × 151936 again and again took 8.6 µs a call, with a line
+// each XXXX.)
+struct alignas(128) AmaxRow {
+  unsigned long long part[ARGMAX_CHUNKS];
+  alignas(128) unsigned count;  // zero between calls
+};
+
 // One launch: each workgroup publishes its chunk's maximum with an agent-coherent store, completed before it counts
 // itself in; the last of the row to arrive reads the sixteen back agent-coherently (the reads are issued under the branch
-// on the count) and resets the count for the next call. 17 × 151936: 8.6 µs against 5.4 + 2.3 and the gap of a second
-// launch (argmax and acceptance as called from a program: 17.8 → 14.4 µs).
+// on the count) and resets the count for the next call. Called again and again, one launch against two: 17 × 151936 6.2
+// against 7.0 µs (8.2 against 8.9 on rows not in a cache), one row 6.0 against 6.5, 5 × 32000 4.5 against 6.3.
 __global__ __launch_bounds__(256) void argmax_kernel(const float* __restrict__ x, int ldx, int N,
-                                                     unsigned long long* __restrict__ part, unsigned* __restrict__ ctr,
-                                                     uint32_t* __restrict__ out) {
+                                                     AmaxRow* __restrict__ rows, uint32_t* __restrict__ out) {
   __shared__ unsigned arrived;
   const int row = blockIdx.x;
+  AmaxRow& r = rows[row];
   float b;
   uint32_t ix;
   argmax_chunk(x, ldx, N, row, blockIdx.y, b, ix);
   if (threadIdx.x == 0) {
-    __hip_atomic_store(part + row * ARGMAX_CHUNKS + blockIdx.y,
+    __hip_atomic_store(r.part + blockIdx.y,
                        (static_cast<unsigned long long>(__float_as_uint(b)) << 32) | ix, __ATOMIC_RELAXED,
                        __HIP_MEMORY_SCOPE_AGENT);
     __builtin_amdgcn_s_waitcnt(0);
-    arrived = __hip_atomic_fetch_add(ctr + row, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    arrived = __hip_atomic_fetch_add(&r.count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   __syncthreads();
   if (arrived != ARGMAX_CHUNKS - 1 || threadIdx.x >= 64) return;
   const int l = threadIdx.x;
-  const unsigned long long v = __hip_atomic_load(part + row * ARGMAX_CHUNKS + min(l, ARGMAX_CHUNKS - 1),
-                                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const unsigned long long v =
+      __hip_atomic_load(r.part + min(l, ARGMAX_CHUNKS - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   argmax_merge(__uint_as_float(unsigned(v >> 32)), unsigned(v), l, out + row);
-  if (l == 0) __hip_atomic_store(ctr + row, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (l == 0) __hip_atomic_store(&r.count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 __global__ __launch_bounds__(64) void argmax_final_kernel(const float2* __restrict__ part, uint32_t* __restrict__ out) {
@@ -256,7 +264,7 @@ int launch_embed_act(ih_ctx* c, const uint32_t* tok, const uint32_t* w, const ui
   return IH_OK;
 }
 
-// Scratch of argmax_kernel for `rows` rows: the chunks' maxima, then one arrival count per row, zero between calls.
+// Scratch of argmax_kernel for `rows` rows, counts zero.
 // Grown on demand, the stream drained before an old buffer is freed.
 static int ensure_argmax(ih_ctx* c, int rows) {
   if (c->amax_rows >= rows) return IH_OK;
@@ -266,7 +274,7 @@ static int ensure_argmax(ih_ctx* c, int rows) {
   c->amax = nullptr;
   c->amax_rows = 0;
   const int cap = std::max(rows, MAX_TOK);
-  const size_t bytes = size_t(cap) * (ARGMAX_CHUNKS * sizeof(unsigned long long) + sizeof(unsigned));
+  const size_t bytes = size_t(cap) * sizeof(AmaxRow);
   if (hipMalloc(&c->amax, bytes) != hipSuccess) return fail(IH_ENOMEM, "argmax scratch allocation failed");
   IH_TRY(fill(c, c->amax, 0, bytes));
   c->amax_rows = cap;
@@ -277,8 +285,7 @@ int launch_argmax(ih_ctx* c, const float* x, int ldx, int rows, int N, uint32_t*
   IH_TRY(ensure_argmax(c, rows));
   TimedLaunch tl(c, TC_ARGMAX, double(rows) * N * 4);
   tlaunch(tl, argmax_kernel, dim3(rows, ARGMAX_CHUNKS), dim3(256), 0, c->stream, x, ldx, N,
-          static_cast<unsigned long long*>(c->amax), reinterpret_cast<unsigned*>(
-              static_cast<unsigned long long*>(c->amax) + size_t(c->amax_rows) * ARGMAX_CHUNKS), out);
+          static_cast<AmaxRow*>(c->amax), out);
   IH_HIP(hipGetLastError());
   return IH_OK;
 }
