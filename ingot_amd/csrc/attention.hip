@@ -533,10 +533,12 @@ __global__ __launch_bounds__(ATT_THREADS) void attn_kernel(AttnArgs a) {
   attn_merge<HD>(a, st, live, kvh, sidx, cls, lt, m0 + (lane & 15), lane, L.ml, L.part());
 }
 
-// Small blocks (at most FEW tiles of queries, e.g. plain decoding): three waves per tile, one per class, each reading
-// its steps' cache bytes straight into the MFMA operand registers: no staging, no barrier before the merge. One row at
-// 611 positions: 4.6 µs against 7.7 in the kernel above, whose 16 waves mostly stage; with three tiles every byte would
-// be read and converted three times.
+// Small blocks: one workgroup per (split, KV head, FEW tiles), three waves per tile, one per class, each reading its steps'
+// cache bytes straight into the MFMA operand registers: no staging, no barrier before the merge. One row at 611
+// positions: 4.6 µs against 7.7 in the kernel above, whose 16 waves mostly stage. More tiles read and convert every byte
+// once per FEW of them; that wins as long as the launch is one workgroup per CU at most, since one of the kernel above
+// then leaves CUs idle or is mostly latency (8 heads per KV head, 4 KV heads of 128, 8 rows: 1000 positions 57.8 → 55.2 µs
+// a layer, 16000 65.2 → 62.2; 12 rows at 1000 65.3 → 62.2, at 2000 in 64-key splits, three workgroups for two CUs, 65.9 → 66.2).
 constexpr int FEW = 2;
 template <int HD, bool RING>
 __global__ __launch_bounds__(64 * NCLS * FEW) void attn_few_kernel(AttnArgs a) {
@@ -547,7 +549,8 @@ __global__ __launch_bounds__(64 * NCLS * FEW) void attn_few_kernel(AttnArgs a) {
   const int sidx = blockIdx.y, kvh = blockIdx.x;  // as in attn_kernel
   if (sidx >= ap.nsplit) return;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int qd = lane >> 4, lt = wave / NCLS, cls = wave % NCLS, m0 = 16 * lt;
+  const int qd = lane >> 4, lt = wave / NCLS, cls = wave % NCLS, m0 = 16 * (FEW * int(blockIdx.z) + lt);
+  const bool live = m0 < a.G * a.B;  // uniform
   const SplitKeys sk = split_keys(a, ap, sidx);
   const size_t hrow = size_t(kvh) * a.vld;
   const unsigned l16 = unsigned(lane & 15) * 64u + unsigned(qd) * 16u;
@@ -581,7 +584,7 @@ __global__ __launch_bounds__(64 * NCLS * FEW) void attn_few_kernel(AttnArgs a) {
   load_k(s, sr);
   attn_tile<HD>(a, kvh, ap.P, m0, lane, qf, mk, st);
   load_v(s);
-  for (; s < sk.nsteps; s += NCLS) {
+  for (; live && s < sk.nsteps; s += NCLS) {
     const int key0 = sk.kbase + STEP * s;
     f32x4 sc[2][2];
 #pragma unroll
@@ -615,7 +618,7 @@ __global__ __launch_bounds__(64 * NCLS * FEW) void attn_few_kernel(AttnArgs a) {
 #pragma unroll
       for (int h = 0; h < 2; ++h) sr[x][h] = sn[x][h];
   }
-  attn_merge<HD>(a, st, true, kvh, sidx, cls, lt, m0 + (lane & 15), lane, sml, part);
+  attn_merge<HD>(a, st, live, kvh, sidx, cls, lt, m0 + (lane & 15), lane, sml, part);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -813,9 +816,10 @@ int launch_attention(ih_ctx* c, const AttnArgs& a) {
   IH_CHECK(qtiles <= 16, IH_EINVAL, "attention: at most 256 query rows per KV head");
   IH_CHECK(a.C > 0 && a.C % STEP == 0, IH_EINVAL, "attention: unsupported key chunk");
   IH_CHECK(size_t(a.vld) * a.HD < (size_t(1) << 31), IH_EINVAL, "attention: a KV head's cache must be below 2 GiB");
-  const bool few = qtiles <= FEW, ring = a.ring != 0;
-  const dim3 grid(a.KVH, a.nsplit, few ? 1 : (qtiles + WTILES - 1) / WTILES);
-  const dim3 block(few ? 64 * NCLS * qtiles : ATT_THREADS);
+  const bool few = qtiles <= FEW || a.KVH * a.nsplit * ((qtiles + FEW - 1) / FEW) <= c->cu_count, ring = a.ring != 0;
+  const int per = few ? FEW : WTILES;
+  const dim3 grid(a.KVH, a.nsplit, (qtiles + per - 1) / per);
+  const dim3 block(few ? 64 * NCLS * std::min(FEW, qtiles) : ATT_THREADS);
   // Algorithmic bytes: the int8 K and V and their fp16 scales of every key the launched splits cover, and q.
   const double keys = double(a.P + a.B) - double(a.s0) * a.C;
   TimedLaunch tl(c, TC_ATTN, double(a.KVH) * keys * (2 * a.HD + 4) + double(a.KVH) * Q * a.HD * 2);

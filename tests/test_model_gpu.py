@@ -22,8 +22,7 @@ GQA8 = dict(n_layers=2, hidden=512, n_q_heads=8, n_kv_heads=1, head_dim=64, inte
 MOE4 = dict(n_layers=1, hidden=256, n_q_heads=4, n_kv_heads=2, head_dim=128, intermediate=0, vocab=1000,
             n_experts=8, top_k=2, expert_intermediate=128, expert_format=0)
 SWA = dict(GQA8, sinks=1, sliding_window=16)
-# Config 1's grouping (4 q heads per KV head): 17 rows make 68 query rows, five 16-row tiles, the fifth shared by
-# four waves of the attention workgroup.
+# Config 1's grouping (4 q heads per KV head): 17 rows make 68 query rows, five 16-row tiles.
 GQA4 = dict(n_layers=2, hidden=512, n_q_heads=8, n_kv_heads=2, head_dim=128, intermediate=256, vocab=1000)
 MOEX = dict(n_layers=1, hidden=192, n_q_heads=8, n_kv_heads=2, head_dim=64, intermediate=0, vocab=777, n_experts=8,
             top_k=4, expert_intermediate=96, expert_format=1, router_bias=1, expert_bias=1, act=1, sinks=1,
@@ -352,9 +351,9 @@ def test_split_k_epilogues_match_the_whole_k_step():
 @pytest.mark.parametrize("shape,chunk", [(GQA4, 0), (GQA4, 160), (GQA8, 32), (GQA8, 0), (SWA, 96), (YARN, 0)],
                          ids=["gqa4-auto", "gqa4-160", "gqa8-32", "gqa8-auto", "swa-96", "yarn-auto"])
 def test_rows_do_not_depend_on_the_attention_kernel(ctx, shape, chunk):
-    """Blocks of at most two 16-query tiles take the small-block attention, larger ones the staged one, models of more
-    than 80 rows two workgroups per split: the leading rows of every block size around those edges are bit-identical to
-    the full block's, at a capacity that ends inside a 32-slot block and with chunks of whole and partial rounds."""
+    """The small-block attention with one to five workgroups of two 16-query tiles per split: the leading rows of every
+    block size around those edges are bit-identical to the full block's, at a capacity that ends inside a 32-slot block
+    and with chunks of whole and partial rounds."""
     P, cap = 596, 613
     d, m, kv = make(ctx, shape, P=P, cap=cap, chunk=chunk)
     try:
@@ -453,3 +452,27 @@ def test_attention_weights_times_the_largest_value_scales(ctx, tmp_path, shape, 
     scale = np.abs(got[4]).max()
     assert np.isfinite(got[16]).all()
     assert np.abs(got[16] - got[4]).max() <= 0.02 + 0.01 * scale
+
+
+# Enough KV heads and splits that blocks of more than two 16-query tiles take the staged attention, not the small-block
+# one: 4 and 8 q heads per KV head, 128 and 64 dims, with a ring and sinks.
+STAGED = dict(n_layers=2, hidden=256, n_q_heads=32, n_kv_heads=8, head_dim=128, intermediate=256, vocab=500)
+STAGED64 = dict(STAGED, n_q_heads=64, head_dim=64, sinks=1, sliding_window=1000)
+
+
+@pytest.mark.parametrize("shape", [STAGED, STAGED64], ids=["gqa4-hd128", "gqa8-hd64-ring-sinks"])
+@pytest.mark.parametrize("chunk", [32, 160, 0])
+def test_rows_do_not_depend_on_the_staged_attention(ctx, shape, chunk):
+    """Blocks on both sides of the rule that picks the attention kernel by its workgroups: the leading rows of every block
+    size are bit-identical to the full block's."""
+    d, m, kv = make(ctx, shape, P=2000, cap=2100, chunk=chunk)
+    try:
+        toks = np.random.default_rng(3).integers(0, d.vocab, size=17).astype(np.uint32)
+        _, full = kv.verify(toks, want_logits=True)
+        assert np.all(np.isfinite(full))
+        for B in (1, 2, 4, 5, 8, 9, 11, 16):
+            _, part = kv.verify(toks[:B], want_logits=True)
+            assert np.array_equal(part.view(np.uint32), full[:B].view(np.uint32)), B
+    finally:
+        kv.free()
+        m.free()
