@@ -629,14 +629,23 @@ int ih_kv_create_chunked(ih_model* m, int capacity, int chunk, ih_kv** out) {
   kv->ctx = m->ctx;
   kv->cap = capacity;
   // Key chunk: fixed per cache, so a row's result is the same for every block size and every position (the splits
-  // are fixed key ranges [s·C, (s+1)·C)). At full capacity the workgroups of all KV heads are one per CU for the model's
-  // largest block (with 128-dim heads a block of more than 80 query rows takes two workgroups per split; 64-dim ones
-  // fit two to a CU), rounded up to whole attention rounds of 96 keys (a
-  // short cache: two thirds of one, more splits being worth more than the third class).
-  const int wgs = d.head_dim == 128 ? (m->Qpad + 79) / 80 : 1;
-  const int per_head = std::max(1, m->ctx->cu_count / std::max(1, d.n_kv_heads * wgs));
-  int C = (capacity + per_head - 1) / per_head;
-  C = C <= 64 ? 64 : (C + 95) / 96 * 96;
+  // are fixed key ranges [s·C, (s+1)·C)). At full capacity the workgroups of all KV heads are one per CU, rounded up to
+  // whole attention rounds of 96 keys, for the model's largest block: one of more than 80 query rows takes two workgroups
+  // per split. With 64-dim heads in longer caches they are counted for the smaller blocks, since a workgroup's stream then
+  // costs more than the second round of a full block (no two of them fit a CU; 64 q and 8 KV heads, µs a layer: 2000
+  // positions, 192 keys against 64, 17 rows 77.5 and 81.3, 8 rows 54.8 and 55.3, one row 45.3 and 44.9; 8000 positions, 576
+  // against 288, 17 rows 82.3 and 85.6, 10 rows 65.3 and 62.8, one row 48.1 and 46.3). A short cache takes two thirds of a
+  // round, more splits being worth more than the third class, unless small blocks no longer fit the CUs in one round then
+  // (32 q and 4 KV heads of 128, 2000 positions: 12 rows 63.0 against 65.9).
+  const int wgs = (m->Qpad + 79) / 80, cus = m->ctx->cu_count;
+  auto fill_cus = [&](int w) {
+    const int per_head = std::max(1, cus / std::max(1, d.n_kv_heads * w));
+    return (capacity + per_head - 1) / per_head;
+  };
+  int C = fill_cus(wgs);
+  if (d.head_dim == 64 && fill_cus(1) > 192) C = fill_cus(1);
+  const bool small = C <= 64 && (wgs == 1 || (capacity + 63) / 64 * d.n_kv_heads * 3 <= cus);
+  C = small ? 64 : (C + 95) / 96 * 96;
   if (chunk) C = chunk;
   kv->chunk = C;
   const int L = d.n_layers, KVH = d.n_kv_heads, HD = d.head_dim;
