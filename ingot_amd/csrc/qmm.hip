@@ -66,10 +66,18 @@ __global__ void pack_int4_kernel(const uint32_t* __restrict__ w, const uint16_t*
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// bf16 rows that are not 16-byte aligned → aligned rows of ld elements. Grid (M), 256 threads.
-__global__ void align_rows_kernel(const uint16_t* __restrict__ x, int ldx, int K, uint16_t* __restrict__ out, int ld) {
-  const int i = blockIdx.x;
-  for (int c = threadIdx.x; c < K; c += blockDim.x) out[size_t(i) * ld + c] = x[size_t(i) * ldx + c];
+// bf16 rows that are not 16-byte aligned → aligned rows of ld elements, one thread per eight (K is a multiple of 64):
+// grid (⌈K / 512⌉, M), 64 threads. (With one workgroup per row and an element per thread and trip, 16 rows at an odd
+// element through 4096 × 4096 took 11.0 µs a call, with this 8.5.)
+__global__ __launch_bounds__(64) void align_rows_kernel(const uint16_t* __restrict__ x, int ldx, int K,
+                                                        uint16_t* __restrict__ out, int ld) {
+  const int i = blockIdx.y, c = 8 * (blockIdx.x * 64 + threadIdx.x);
+  if (c >= K) return;
+  const uint16_t* p = x + size_t(i) * ldx + c;
+  unsigned w[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) w[e] = unsigned(p[2 * e]) | unsigned(p[2 * e + 1]) << 16;
+  *reinterpret_cast<uint4*>(out + size_t(i) * ld + c) = make_uint4(w[0], w[1], w[2], w[3]);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -330,7 +338,7 @@ int launch_qmm_rows(ih_ctx* c, const ih_qmat* W, const uint16_t* x, int ldx, int
       (size_t(M - 1) * ldx + W->K) * 2 >= (size_t(1) << 31)) {
     IH_TRY(ensure_act(c, c->act, W->K, false));
     uint16_t* rows = static_cast<uint16_t*>(c->act.frag);
-    align_rows_kernel<<<M, 256, 0, c->stream>>>(x, ldx, W->K, rows, W->nkb * KBLK);
+    align_rows_kernel<<<dim3((W->K + 511) / 512, M), 64, 0, c->stream>>>(x, ldx, W->K, rows, W->nkb * KBLK);
     IH_HIP(hipGetLastError());
     x = rows;
     ldx = W->nkb * KBLK;
