@@ -284,7 +284,7 @@ def run_config(ctx, config: str, steps: int, warmup: int, profile: bool, cpu: bo
         for i in range(steps):
             step(i)
         ctx.sync()
-        names = ["qmm", "attention", "attn_prework", "attn_reduce", "rows", "argmax", "moe", "other", "qmm_finish"]
+        names = ["qmm", "attention", "attn_prework", "attn_reduce", "rows", "argmax", "moe", "other"]
         for c, n in enumerate(names):
             t = C.c_double()
             cnt = C.c_int()

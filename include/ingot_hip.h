@@ -255,12 +255,13 @@ int ih_model_free(ih_model* model);
 size_t ih_model_weight_bytes(const ih_model* model);
 
 /* An int8 KV cache for `capacity` positions (int8 K and V per KV head, fp16 scale per token and head). The attention
- * key chunk is fixed per cache (256 … 2048 keys, from the capacity) so a row's result is the same for every block
- * size. AttentionLayer's kc/vt/ks/vs (Sources/Ingot/Layers/Attention.swift:272-390). */
+ * key chunk is fixed per cache (from the capacity: 64 keys in a short cache, else a multiple of 96) so a row's result is
+ * the same for every block size. AttentionLayer's kc/vt/ks/vs (Sources/Ingot/Layers/Attention.swift:272-390). */
 int ih_kv_create(ih_model* model, int capacity, ih_kv** out);
 /* The same with an explicit key chunk C (a positive multiple of 32; 0 = automatic). Attention splits the keys into the
  * fixed ranges [s·C, (s+1)·C) and merges them in order (pattn_i8 chunks, Attention.swift:389-390); the automatic C
- * gives one workgroup per CU over all KV heads at full capacity. */
+ * gives about one workgroup per CU over all KV heads at full capacity, for the model's largest block (two workgroups per
+ * split above 80 query rows; in longer caches of 64-dim heads for the smaller blocks). */
 int ih_kv_create_chunked(ih_model* model, int capacity, int chunk, ih_kv** out);
 /* Frees a cache. A cache whose model was freed first refuses calls that need the model (IH_EINVAL) and can still be
  * freed. */

@@ -115,7 +115,7 @@ struct ih_qmat {
 namespace ih {
 // Per-kernel-class timing (ih_timing_*): events recorded around each launch when enabled.
 enum TimingClass : int { TC_QMM = 0, TC_ATTN = 1, TC_PREWORK = 2, TC_REDUCE = 3, TC_ROWS = 4, TC_ARGMAX = 5, TC_MOE = 6,
-                         TC_OTHER = 7, TC_QMM_FINISH = 8, TC_COUNT = 9 };
+                         TC_OTHER = 7, TC_COUNT = 8 };
 struct TimingRec {
   int cls;
   double bytes;

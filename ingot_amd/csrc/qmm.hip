@@ -284,7 +284,6 @@ int launch_qmm_ex(ih_ctx* c, const ih_qmat* W, int expert, const ActBuf& a, int 
   p.xa = static_cast<const uint4*>(a.frag);
   p.y = ep.y;
   p.ldy = ep.ldy;
-  p.mode = ep.mode;
   if (ep.mode == QM_F32_SCALE || ep.mode == QM_GLU_ACT) {
     IH_CHECK(a.ss && a.nss > 0, IH_EINVAL, "qmm: the input activation carries no RMSNorm sums");
     p.ss_in = a.ss;
@@ -347,7 +346,6 @@ int launch_qmm_rows(ih_ctx* c, const ih_qmat* W, const uint16_t* x, int ldx, int
   p.ldx = ldx;
   p.y = y;
   p.ldy = ldy;
-  p.mode = out_mode;
   TimedLaunch tl(c, TC_QMM, double(W->algo_bytes) + double(M) * W->K * 2 +
                                 double(M) * W->N * (out_mode == QM_BF16 ? 2 : out_mode == QM_F32_ADD ? 8 : 4));
   IH_CHECK(qmm_rows_dispatch(tl, sh, grid, c->stream, p, M, out_mode), IH_EINVAL, "qmm: launch shape not instantiated");

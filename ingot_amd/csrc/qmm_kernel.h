@@ -14,7 +14,7 @@ struct QmmParams {
   const uint4* xa;         // activation fragments, or (XN) bf16 rows of ldx elements
   int ldx, K;              // XN
   void* y;
-  int ldy, M, N, Npad, nkb, mode;
+  int ldy, M, N, Npad, nkb;
   // The nibble-decode constants 0x000F000F and 0x43004300, passed as arguments so that they live in SGPRs and the
   // compiler can use the three-operand v_and_or_b32 (gfx9 VOP3 takes no literal constants).
   unsigned kmask, kbias;
