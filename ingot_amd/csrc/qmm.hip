@@ -115,7 +115,9 @@ static QmmShape qmm_shape(int Npad, int nkb, int M) {
 // Products of the caller's rows whose K-block count no exact shape tiles: the smallest span of the row-tile class that
 // covers K (waves past the end idle), or the largest one in as many splits as it takes. One wave per workgroup and
 // K-block, the general shape below, leaves the sum of all the splits to the last workgroup (2880 × 4160: 15.8 µs in two
-// launches against 5).
+// launches against 5). Four row tiles are taken from 2048 on (vocabulary-sized N), where they were measured first. Below,
+// down to 513, they are faster for most sizes as well (17 rows, two against four: 8256 × 1600 8.1 and 6.4 µs, 11008 × 4160
+// 14.6 and 13.3, 32000 × 4160 28.3 and 26.2, but 24576 × 4160 21.8 and 25.7; at 384 tiles 8.2 and 13.0).
 static QmmShape qmm_shape_ragged(int Npad, int nkb) {
   static constexpr int one[5][2] = {{16, 1}, {16, 2}, {16, 3}, {16, 4}, {14, 8}};
   static constexpr int two[4][2] = {{16, 1}, {16, 2}, {16, 4}, {14, 8}};  // (16, 3) spills with two row tiles
