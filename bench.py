@@ -454,7 +454,7 @@ def config0(ctx) -> dict:
             "qmm_kernel_us": round(kernel_us, 2), "qmm_kernel_gbs": round(algo / (kernel_us * 1e3), 1),
             "qmm_back_to_back_us": round(b2b_us, 2), "qmm_back_to_back_gbs": round(algo / (b2b_us * 1e3), 1),
             "qmm_algorithmic_bytes": algo,
-            "note": "a call = bf16 rows to the activation layout + the qmm launch",
+            "note": "a call = one qmm launch that reads the bf16 rows itself",
             "argmax_accept_us": round(acc_us, 2), "accepted_m": m,
             "argmax_equal": bool(np.array_equal(gpu_top, top))}
 

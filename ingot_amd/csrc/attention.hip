@@ -15,14 +15,16 @@
 // fragments in LDS, two rounds of loads in flight). Sᵀ = K·Qᵀ (v_mfma_f32_16x16x32_f16, keys as rows so each lane holds
 // 4 keys of one query), online softmax in base 2 per query column, P stays in registers as the B operand of
 // Oᵀ += Vᵀ·Pᵀ. The classes are merged in LDS; a split writes O/l in fp16 with its (reference, sum) and the reduction
-// merges the splits in a fixed order. Blocks of at most 32 query rows take a kernel of three waves per tile that reads
-// the cache straight into MFMA operands (attn_few_kernel); both run the same attn_step and attn_merge. A query's result
+// merges the splits in a fixed order. Blocks of at most 32 query rows, and larger ones whose tiles in pairs are at most one
+// workgroup per CU, take a kernel of three waves per tile that reads the cache straight into MFMA operands
+// (attn_few_kernel); both run the same attn_step and attn_merge. A query's result
 // does not depend on the other rows of the block: steps and classes are counted from fixed key positions, the split
 // boundaries are fixed multiples of C, and every row is reduced in the same order whatever tile it falls in.
 //
-// What bounds it: a 1056-key split of 80 rows (32K positions, 8 KV heads of 128) spends, per 128 keys, ≈ 1.1 µs on its
-// HBM stream (≈ 30 GB/s per CU), ≈ 1.3 µs of VALU issue (conversion, softmax), ≈ 0.9 µs of LDS reads and ≈ 0.5 µs of
-// MFMA, which overlap to ≈ 2.4 µs, after ≈ 6 µs of launch, first loads and merge. One tile per wave at 16 waves (four
+// What bounds it: no one unit. A 1056-key split of 80 rows (32K positions, 8 KV heads of 128, 27.5 µs) by its counters: a
+// wave lives 22.5 µs, in which a SIMD's vector ALU is busy for 11.9 (conversion, softmax), a CU's LDS for 11.3 (no bank
+// conflicts), a SIMD's matrix core for 4.3, and the HBM stream takes 9.9 at 6.9 TB/s; the rest is the wait for the first
+// loads and the merge, during which none of them works. One tile per wave at 16 waves (four
 // per SIMD, 128 VGPRs) overlaps them better than two or three tiles per wave at eight (28.7 against 33.2 µs, and
 // 54.5 → 32.7 µs with 64-dim heads over 64K positions, where one wave per tile left three SIMDs with one tile).
 

@@ -597,7 +597,8 @@ int launch_gather(ih_ctx* c, const ih_qmat* W, const GatherParams& base, int slo
   // beats two waves over four tiles (3.30), over two tiles (3.72) and four waves over two (3.95) or one (5.13). With more
   // K-blocks four waves over two tiles beat two waves (MXFP4, K = 2880, 32 experts top-4: 5760 rows, 5 and 9 rows a block,
   // 27.2 and 36.0 against 29.0 and 38.2 µs; 2880 rows 17.5 and 20.4 against 18.2 and 20.0, one row 9.3 against 12.1, 17
-  // rows 24.4 against 27.8). A slot holds few pairs, so a workgroup's life is a few memory latencies and the rate is set by
+  // rows 24.4 against 27.8; inside the model, 9 rows and weights from HBM, 2880 rows 21.6 against 20.3: the price of one order
+  // for every block there). A slot holds few pairs, so a workgroup's life is a few memory latencies and the rate is set by
   // how much each wave streams behind them: longer waves win until the registers cost waves per SIMD (eight tiles: 171
   // VGPRs, 3.53 ms; a ring of two or three stages: 4.47, 5.70). A single slot (a router, or one expert) has few
   // workgroups; every K-block of a wave, up to four, is requested at entry there, and K is split in two where the launch
