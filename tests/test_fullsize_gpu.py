@@ -100,8 +100,8 @@ def test_fullsize_verify_matches_oracle(ctx, name):
         near_ties = int(np.sum(~sure))
         near_tie_flips = int(np.sum(top1[~sure] != ref_top1[~sure]))
         # How far the oracle moves when its attention rounds p·vs to fp16, as the reference and the GPU do, reported next
-        # to the error (configs 3 and 4: 0.020 and 0.115 against GPU errors of 0.021 and 0.13 at logit scales of 42 and
-        # 44), and the GPU's distance from that variant (0.022 and 0.114: no closer — its own fp16 roundings are another
+        # to the error (configs 3 and 4: 0.020 and 0.115 against GPU errors of 0.022 and 0.16 at logit scales of 42 and
+        # 44), and the GPU's distance from that variant (0.022 and 0.113: hardly closer — its own fp16 roundings are another
         # draw of the same size).
         with oracle.attn_p16():
             p16_logits, _ = om.verify(toks)
